@@ -5,6 +5,7 @@
 
 #include "ckfft/ckfft_gpu.h"
 #include "ckfft_internal.h"
+#include "fft_outputs.h"
 
 namespace ckfft_gpu {
 
@@ -52,7 +53,8 @@ struct BatchBuild {
     int n_wide = 0;                   // items of the wide kernel's queue
     std::vector<BatchTransform> trs;  // the persistent kernel's transforms, by class
     std::vector<BatchExtra> extras;
-    // complex 2^16 transforms run by the table pass launches, forward then inverse
+    // complex 2^16 transforms run by the table pass launches, forward then inverse; none of their outputs
+    // is written by another transform that may run beside them
     std::vector<BatchTransform> pass_fwd, pass_inv;
     long long bytes = 0;              // algorithmic bytes of the whole batch
     int persistent = 0;               // transforms taken by the persistent kernel
@@ -61,6 +63,8 @@ struct BatchBuild {
 // Validation of one descriptor (single-signal rules, plus device buffers when asked);
 // false records the reason for CkFftBatchLastError.
 bool batch_check_desc(const CkFftContext* ctx, const CkFftBatchDesc& d, int index, bool check_pointers);
+// The memory a transform writes.
+OutputRange output_range(const CkFftBatchDesc& d);
 // Validate and group a batch; var_override >= 0 forces one thread layout for every class.
 // narrow (batch plans): classes the narrow persistent kernel takes (two workgroups per CU) go
 // to its queue, and the context's tuning may send complex 2^16 transforms to ordinary launches;

@@ -274,6 +274,15 @@ long long transform_bytes(int kind, int log2n)
     return (kind == kRealForward || kind == kRealInverse) ? 4 * n + 8 * (n / 2 + 1) : 16 * n;
 }
 
+OutputRange output_range(const CkFftBatchDesc& d)
+{
+    const uintptr_t begin = (uintptr_t)d.output;
+    const size_t bytes = d.kind == kRealForward   ? sizeof(float2) * ((size_t)d.n / 2 + 1)
+                         : d.kind == kRealInverse ? sizeof(float) * (size_t)d.n
+                                                  : sizeof(float2) * (size_t)d.n;
+    return OutputRange{begin, begin + bytes};
+}
+
 bool batch_check_desc(const CkFftContext* ctx, const CkFftBatchDesc& d, int index, bool check_pointers)
 {
     if (d.kind < 0 || d.kind > 3) return batch_invalid("bad kind", index);
@@ -297,6 +306,7 @@ bool batch_build(const CkFftContext* ctx, const CkFftBatchDesc* descs, int count
         int kind, log2n, logc, idx;
     };
     std::vector<Entry> pers;
+    std::vector<int> passes, extras;   // descriptors of the table passes and of ordinary launches
     pers.reserve(count);
     for (int i = 0; i < count; ++i) {
         const CkFftBatchDesc& d = descs[i];
@@ -312,15 +322,35 @@ bool batch_build(const CkFftContext* ctx, const CkFftBatchDesc* descs, int count
         // the table passes keep their intermediate in the output, so they need separate buffers
         if (is_twopass && !(narrow && ctx->tune[d.kind][kPassLogN] == 2) &&
             !buffers_overlap(d.input, sizeof(float2) << kPassLogN, d.output, sizeof(float2) << kPassLogN)) {
-            (d.kind == kComplexInverse ? out.pass_inv : out.pass_fwd)
-                .push_back(BatchTransform{(const float2*)d.input, (float2*)d.output});
+            passes.push_back(i);
         } else if (ok && !is_twopass) {
             pers.push_back({d.kind, log2n, logc, i});
         } else {
-            out.extras.push_back(BatchExtra{(Kind)d.kind, log2n, d.input, d.output});
+            extras.push_back(i);
         }
         out.bytes += transform_bytes(d.kind, log2n);
     }
+    // Nor may another transform write there meanwhile: one whose output others share goes to the
+    // ordinary launches, which come one after another behind all that runs side by side (in a plan the table
+    // passes run beside the persistent launches, in a server behind them).
+    if (!passes.empty()) {
+        std::vector<OutputRange> held, others;
+        for (int i : passes) held.push_back(output_range(descs[i]));
+        if (narrow)
+            for (const Entry& e : pers) others.push_back(output_range(descs[e.idx]));
+        const std::vector<char> shared = shared_outputs(held, others);
+        for (size_t k = 0; k < passes.size(); ++k) {
+            const CkFftBatchDesc& d = descs[passes[k]];
+            if (shared[k])
+                extras.push_back(passes[k]);
+            else
+                (d.kind == kComplexInverse ? out.pass_inv : out.pass_fwd)
+                    .push_back(BatchTransform{(const float2*)d.input, (float2*)d.output});
+        }
+        std::sort(extras.begin(), extras.end());   // descriptor order
+    }
+    for (int i : extras)
+        out.extras.push_back(BatchExtra{(Kind)descs[i].kind, ilog2(descs[i].n), descs[i].input, descs[i].output});
     // group by class, keep descriptor order within a class
     std::stable_sort(pers.begin(), pers.end(), [](const Entry& a, const Entry& b) {
         return a.kind != b.kind ? a.kind < b.kind : a.logc < b.logc;

@@ -77,6 +77,7 @@ struct Slot {
     float2* d_scratch = nullptr;
     size_t scratch_bytes = 0;
     std::vector<long long> reqs;
+    BatchOutputs outputs;                // what the batch in flight writes
     long long bytes = 0;
     bool busy = false;
 };
@@ -173,6 +174,14 @@ void finish_slot(CkFftServer* S, Slot& sl, bool ok)
     S->cv.notify_all();
 }
 
+// Whether a request keeps its intermediate in its output: the multi-pass sizes, and in the split-BF16x3
+// mode those of two passes there (2^15 and 2^16).
+bool holds_intermediate(const CkFftContext* ctx, const CkFftBatchDesc& d)
+{
+    const int n_max = 1 << (d.kind >= kRealForward ? kLogMaxLds + 1 : kLogMaxLds);   // of one workgroup
+    return d.n > n_max || (ctx->precision == kCkFftPrecision_SplitBf16x3 && d.kind < kRealForward && d.n == n_max);
+}
+
 // `descs` and `bytes` were copied from the requests `batch` under the lock (the request
 // deque may grow concurrently, so it is only indexed under the lock).
 bool launch_batch(CkFftServer* S, Slot& sl, std::vector<long long>& batch, const std::vector<CkFftBatchDesc>& descs,
@@ -183,11 +192,18 @@ bool launch_batch(CkFftServer* S, Slot& sl, std::vector<long long>& batch, const
     if (!batch_build(S->ctx, descs.data(), (int)descs.size(), -1, false, b, false)) return false;
     const DeviceTables tb = context_tables(S->ctx);
     bool ok = true;
-    if (!b.items.empty() && b.items.size() <= (size_t)kInlineQueue && b.trs.size() <= (size_t)kInlineQueue) {
+    // A batch that writes where a transform in flight keeps its intermediate, or the other way round (the same
+    // request again, say), comes after that batch.
+    sl.outputs.clear();
+    for (const CkFftBatchDesc& d : descs) sl.outputs.add(output_range(d), holds_intermediate(S->ctx, d));
+    for (Slot& o : S->slots)
+        if (ok && &o != &sl && o.busy && BatchOutputs::conflict(sl.outputs, o.outputs))
+            ok = serr(hipStreamWaitEvent(sl.stream, o.done, 0), "order after a batch with the same output");
+    if (ok && !b.items.empty() && b.items.size() <= (size_t)kInlineQueue && b.trs.size() <= (size_t)kInlineQueue) {
         // small batch: the queue travels in the launch arguments
         ok = serr(launch_persistent_inline(b, sl.d_ctl, std::min(S->grid, (int)b.items.size()), tb, sl.stream),
                   "persistent launch");
-    } else if (!b.items.empty()) {
+    } else if (ok && !b.items.empty()) {
         const size_t items_bytes = sizeof(BatchItem) * b.items.size();
         const size_t trs_off = (items_bytes + 255) & ~(size_t)255;
         const size_t total = trs_off + sizeof(BatchTransform) * b.trs.size();

@@ -35,6 +35,12 @@ int CkFftRealForwardBatch(CkFftContext* context, int n, int count,
 int CkFftRealInverseBatch(CkFftContext* context, int n, int count,
                           const CkFftComplex* input, float* output, void* stream);
 
+/* An output is the transform's own until the work has ended: larger sizes (complex n >= 2^15, real
+ * n >= 2^16) keep intermediate values there.  Transforms that may run at the same time -- calls
+ * on different streams or from different threads, plans or servers -- must not write to the same
+ * memory, not even the same values.  Transforms of one plan, and requests to one server, may: the
+ * library runs them one after another where it matters. */
+
 /* ---- a batched call that allocates nothing ------------------------------------------
  *
  * No counterpart in the reference.  For callers that cannot allocate device memory: code
@@ -61,7 +67,8 @@ int CkFftTransformBatchNoAlloc(CkFftContext* context, int kind, int n, int count
  * LDS, one with two workgroups per CU for the rest.  Complex 2^16 transforms run as two
  * table-driven pass launches over all of them, both directions (every workgroup of the
  * GPU on one transform's tiles at a time), and transforms the persistent kernels do not take
- * (complex n <= 1, real n <= 4, any n above 2^16) run as ordinary launches; all on the same
+ * (complex n <= 1, real n <= 4, any n above 2^16, complex 2^16 whose output overlaps its input or
+ * another transform's output) run as ordinary launches, one after another on the same
  * stream after the persistent launches.  CkFftBatchInfo reports how many transforms each
  * route takes.
  * Results are bit-identical to the single-signal calls for every transform.
