@@ -15,7 +15,7 @@ __device__ __forceinline__ void report_done(unsigned* done, unsigned ticket)
     if (threadIdx.x == 0) __hip_atomic_store(done, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Input in host memory.  Nothing waited for the stream since the last call on this memory, so the runtime may
+// Input in coherent host memory (the staging slot's) or in this device's own.  Nothing waited for the stream since the last call on this memory, so the runtime may
 // leave the system-scope acquire out of the launch.  Up to two waves acquire by a fence at the kernel's start;
 // the loads of larger groups go past the caches by themselves, as a fence in every wave, which drops the
 // caches' lines of host memory again and again, cost 2 us a call at real 8192 and 4 at 65536 (fence / such

@@ -54,13 +54,17 @@ struct Slot {
 
 enum MemKind { kHostPageable, kHostPinned, kDevice };
 
-MemKind classify(const void* p)
+// own: device memory of the current device itself, neither managed nor another device's.
+MemKind classify(const void* p, bool* own = nullptr)
 {
     hipPointerAttribute_t a;
+    if (own) *own = false;
     if (hipPointerGetAttributes(&a, p) != hipSuccess) {
         (void)hipGetLastError();   // plain pageable host memory is unknown to HIP
         return kHostPageable;
     }
+    int device = -1;
+    if (own && a.type == hipMemoryTypeDevice) *own = hipGetDevice(&device) == hipSuccess && a.device == device;
     if (a.type == hipMemoryTypeDevice || a.type == hipMemoryTypeManaged) return kDevice;
     if (a.type == hipMemoryTypeHost) return kHostPinned;
     return kHostPageable;
@@ -191,22 +195,27 @@ bool reported(const Slot* s)
     }
 }
 
-hipError_t run_direct(Slot* s, Kind kind, int log2n, const void* in, size_t ib, MemKind kin, void* out, size_t ob,
-                      MemKind kout, const DeviceTables& tb)
+hipError_t run_direct(Slot* s, Kind kind, int log2n, const void* in, size_t ib, MemKind kin, bool own, void* out,
+                      size_t ob, MemKind kout, const DeviceTables& tb)
 {
     const size_t ib_al = (ib + 255) & ~size_t(255);
     const void* src = in;
     void* dst = out;
-    if (kin == kHostPageable) {
+    // The output in the slot's own pinned memory: nothing but this call waits for it, so the kernel's
+    // word is enough.  A caller's pinned or device buffer is only handed back with the stream idle.
+    // Without that wait between calls the input must not come from a cache either: the slot's buffer is coherent
+    // memory, and the current device's own memory every launch reads as it is; a caller's pinned memory may
+    // be non-coherent, so it is copied (real 1024, pinned to pageable: 10.6 us a call in place, 10.8 copied, 17.3
+    // with the wait), and managed memory or another device's waits for the stream.
+    const bool word = kout == kHostPageable && signal_supported(kind, log2n) && (kin != kDevice || own);
+    if (kin == kHostPageable || (word && kin == kHostPinned)) {
         std::memcpy(s->h_buf, in, ib);
         src = s->h_buf;
     }
     if (kout == kHostPageable) dst = s->h_buf + ib_al;
     hipError_t e;
     bool ended = false;
-    // The output in the slot's own pinned memory: nothing but this call waits for it, so the kernel's
-    // word is enough.  A caller's pinned or device buffer is only handed back with the stream idle.
-    if (kout == kHostPageable && signal_supported(kind, log2n)) {
+    if (word) {
         e = launch_signal(kind, log2n, src, dst, tb, s->stream, s->done, ++s->ticket);
         ended = e == hipSuccess && reported(s);
     } else {
@@ -222,13 +231,13 @@ hipError_t run_direct(Slot* s, Kind kind, int log2n, const void* in, size_t ib, 
     return e;
 }
 
-hipError_t run_staged(Slot* s, Kind kind, int log2n, const void* in, size_t ib, MemKind kin, void* out, size_t ob,
-                      MemKind kout, const DeviceTables& tb)
+hipError_t run_staged(Slot* s, Kind kind, int log2n, const void* in, size_t ib, MemKind kin, bool own, void* out,
+                      size_t ob, MemKind kout, const DeviceTables& tb)
 {
     const size_t ib_al = (ib + 255) & ~size_t(255);
     hipError_t e = grow(s, ib_al + ob);
     if (e != hipSuccess) return e;
-    if (one_pass(kind, log2n, tb)) return run_direct(s, kind, log2n, in, ib, kin, out, ob, kout, tb);
+    if (one_pass(kind, log2n, tb)) return run_direct(s, kind, log2n, in, ib, kin, own, out, ob, kout, tb);
     char* d_in = s->d_buf;
     char* d_out = s->d_buf + ib_al;
     // input
@@ -273,7 +282,8 @@ hipError_t run_staged(Slot* s, Kind kind, int log2n, const void* in, size_t ib, 
 hipError_t staged_transform(StagingPool* pool, Kind kind, int log2n, const void* in, size_t ib, void* out, size_t ob,
                             const DeviceTables& tb)
 {
-    const MemKind kin = classify(in), kout = classify(out);
+    bool own = false;
+    const MemKind kin = classify(in, &own), kout = classify(out);
     if (kin == kDevice && kout == kDevice) {
         // the calling thread's own default stream: calls from several threads sharing a
         // context (inc/ckfft/ckfft.h:39-41) overlap on the device instead of queueing on
@@ -288,7 +298,7 @@ hipError_t staged_transform(StagingPool* pool, Kind kind, int log2n, const void*
     hipError_t e = hipSuccess;
     Slot* s = acquire(pool, &e);
     if (!s) return e;
-    e = run_staged(s, kind, log2n, in, ib, kin, out, ob, kout, tb);
+    e = run_staged(s, kind, log2n, in, ib, kin, own, out, ob, kout, tb);
     release(pool, s);
     return e;
 }

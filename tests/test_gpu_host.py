@@ -48,3 +48,25 @@ def test_pageable_calls(torch, ctx, kind, log2n):  # noqa: F811
     assert one(n, np.ascontiguousarray(x[3]), got) == 1
     assert np.array_equal(got.view(np.int32), want[3])
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("kind,log2n", [("cfwd", 3), ("rinv", 6), ("rfwd", 10), ("cinv", 13), ("rfwd", 16)])
+def test_pinned_input_rewritten_between_calls(torch, ctx, kind, log2n):  # noqa: F811
+    n, count = 1 << log2n, 12
+    x = torch.from_numpy(make_input(kind, n, count, 0x917 + log2n))
+    length = out_len(kind, n)
+    batch, one = calls(ctx, kind, n)
+    xd = x.cuda()
+    want = torch.empty(count, length, device="cuda")
+    for i in range(count):
+        assert batch(n, 1, xd[i], want[i]) == 1
+    torch.cuda.synchronize()
+    want = want.cpu().numpy().view(np.int32)
+    pinned = torch.empty(x[0].numel(), pin_memory=True)
+    pinned_out = torch.empty(length, pin_memory=True)
+    got = np.empty(length, np.float32)
+    for i in range(count):                      # pinned to pageable, pinned to pinned every third time
+        pinned.copy_(x[i])
+        out = pinned_out if i % 3 == 2 else got
+        assert one(n, pinned, out) == 1
+        assert np.array_equal((pinned_out.numpy() if i % 3 == 2 else got).view(np.int32), want[i]), i

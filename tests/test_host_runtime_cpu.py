@@ -25,3 +25,7 @@ def run(tmp_path, test, source):
 
 def test_server_orders_batches_that_share_an_output(tmp_path):
     run(tmp_path, "serve_outputs", "fft_serve.cpp")
+
+
+def test_host_memory_calls(tmp_path):
+    run(tmp_path, "staging_calls", "fft_staging.cpp")
