@@ -113,5 +113,23 @@ int main()
     c = one(pool, in.data(), out.data());
     CHECK(c.signal == 1 && c.sync == 0);
     staging_destroy(pool);
+    // a size's inverse finds room in its forward's buffers (real n: 4n in, 4n + 8 out, and the other way round)
+    for (int log2n = 4; log2n <= 20; ++log2n) {
+        const size_t n = (size_t)1 << log2n;
+        std::vector<float> a(2 * n), b(2 * n);
+        DeviceTables tb{};
+        for (int kind : {kRealForward, kRealInverse}) {
+            StagingPool* p = staging_create();
+            const auto go = [&](int k) {
+                const size_t ib = k == kRealForward ? 4 * n : 4 * n + 8, ob = k == kRealForward ? 4 * n + 8 : 4 * n;
+                CHECK(staged_transform(p, (Kind)k, log2n, a.data(), ib, b.data(), ob, tb) == hipSuccess);
+            };
+            go(kind);
+            const int dev = count_calls("hipMalloc"), host = count_calls("hipHostMalloc");
+            go(kind == kRealForward ? kRealInverse : kRealForward);
+            CHECK(count_calls("hipMalloc") == dev && count_calls("hipHostMalloc") == host);
+            staging_destroy(p);
+        }
+    }
     return 0;
 }
