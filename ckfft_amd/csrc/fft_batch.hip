@@ -440,6 +440,10 @@ struct _CkFftBatchPlan {
     BatchTransform* d_pass = nullptr;   // table pass transforms: forward ones, then inverse
     int n_pass_fwd = 0, n_pass_inv = 0;
     std::vector<BatchExtra> extras;
+    // Intermediate of the complex 2^16 transforms among the extras whose buffers overlap: they run one after
+    // another, so one serves them all and an execution allocates nothing for them.
+    void* d_scratch = nullptr;
+    size_t scratch_bytes = 0;
     // The table passes and the narrow launch run beside the wide one, each on a stream of
     // the plan's own (created when a plan has two or more of the three launch groups),
     // forked from the caller's stream and joined back into it.
@@ -477,6 +481,13 @@ CkFftBatchPlan* plan_create(CkFftContext* ctx, const CkFftBatchDesc* descs, int 
             !batch_error(hipMemcpy(plan->d_pass, table.data(), sizeof(BatchTransform) * table.size(),
                                    hipMemcpyHostToDevice), "upload pass table"))
             goto bad;
+    }
+    for (const BatchExtra& e : plan->extras) {
+        const size_t bytes = transform_scratch_bytes(e.kind, e.log2n, 1, context_tables(ctx));
+        if (e.log2n != kPassLogN || !bytes || !buffers_overlap(e.in, bytes, e.out, bytes)) continue;
+        if (!batch_error(hipMalloc(&plan->d_scratch, bytes), "hipMalloc(scratch)")) goto bad;
+        plan->scratch_bytes = bytes;
+        break;
     }
     if (plan->n_items) {
         if (!batch_error(hipMalloc(&plan->d_items, sizeof(BatchItem) * b.items.size()), "hipMalloc(items)") ||
@@ -605,8 +616,13 @@ int CkFftBatchPlanExecute(CkFftBatchPlan* plan, void* stream)
         }
     }
     const DeviceTables tb = context_tables(plan->ctx);
-    for (const auto& e : plan->extras)
-        if (!batch_error(launch_transform(e.kind, e.log2n, 1, e.in, e.out, tb, s), "extra launch")) return 0;
+    for (const auto& e : plan->extras) {
+        const bool fits = transform_scratch_bytes(e.kind, e.log2n, 1, tb) <= plan->scratch_bytes;
+        if (!batch_error(launch_transform(e.kind, e.log2n, 1, e.in, e.out, tb, s, fits ? plan->d_scratch : nullptr,
+                                          fits ? plan->scratch_bytes : 0),
+                         "extra launch"))
+            return 0;
+    }
     return 1;
 }
 
@@ -626,6 +642,7 @@ void CkFftBatchPlanDestroy(CkFftBatchPlan* plan)
     if (plan->d_trs) (void)hipFree(plan->d_trs);
     if (plan->d_ctl) (void)hipFree(plan->d_ctl);
     if (plan->d_pass) (void)hipFree(plan->d_pass);
+    if (plan->d_scratch) (void)hipFree(plan->d_scratch);
     for (int i = 0; i < 2; ++i) {
         if (plan->branch[i]) (void)hipStreamDestroy(plan->branch[i]);
         if (plan->join[i]) (void)hipEventDestroy(plan->join[i]);

@@ -149,3 +149,66 @@ def test_first_pass_reads(torch, C, kind, log2n, most):  # noqa: F811
             assert float((y[0].double() - exact).norm() / exact.norm()) <= TOL_FP64
         assert torch.equal(y.view(torch.int32), want[:count].view(torch.int32))
     assert torch.equal(x, keep)
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_plan_of_overlapping_buffers(torch, C, graph):  # noqa: F811
+    """Complex 2^16 transforms whose input and output overlap, beside others: the bits of separate
+    buffers, no memory allocated by an execution, and captured in a caller's graph, replayed."""
+    n = 1 << 16
+    gen = torch.Generator(device="cuda").manual_seed(0x0F)
+    x = torch.randn((4, 2 * n), device="cuda", generator=gen)
+
+    def make(c):
+        buf = torch.zeros((3, 3 * n), device="cuda")
+        y = torch.zeros((2, 2 * n), device="cuda")
+        descs = [(C.kCkFftKind_ComplexForward, n, buf[0], buf[0][n:]), (C.kCkFftKind_ComplexInverse, n, buf[1][n:], buf[1]),
+                 (C.kCkFftKind_ComplexForward, n, buf[2], buf[2][n:]), (C.kCkFftKind_ComplexForward, n, x[3], y[0]),
+                 (C.kCkFftKind_RealForward, 4096, x[3], y[1])]
+        return C.BatchPlan(c, descs, graph=graph), buf, y
+
+    def fill(buf, scale):
+        buf[0][:2 * n] = x[0] * scale
+        buf[1][n:] = x[1] * scale
+        buf[2][:2 * n] = x[2] * scale
+
+    with C.Context(n) as c, C.Context(n) as fresh:
+        want = torch.empty((4, 2 * n), device="cuda")
+        for i in range(4):
+            assert call(c, "cinv" if i == 1 else "cfwd")(n, 1, x[i], want[i]) == 1
+        plan, buf, y = make(c)                        # loads the code
+        assert plan.execute() == 1
+        torch.cuda.synchronize()
+        plan.close()
+        plan, buf, y = make(fresh)
+        info = plan.info()
+        assert info["pass_transforms"] == 1 and info["extra_launches"] == 3
+
+        def check(scale):
+            # scaling by a power of two scales every bit exactly
+            assert torch.equal(buf[0][n:].view(torch.int32), (want[0] * scale).view(torch.int32))
+            assert torch.equal(buf[1][:2 * n].view(torch.int32), (want[1] * scale).view(torch.int32))
+            assert torch.equal(buf[2][n:].view(torch.int32), (want[2] * scale).view(torch.int32))
+            assert torch.equal(y[0].view(torch.int32), want[3].view(torch.int32))
+
+        if graph:                                     # the plan's own graph is made by its first execution
+            assert plan.execute() == 1
+        fill(buf, 1.0)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        assert plan.execute() == 1
+        torch.cuda.synchronize()
+        assert torch.cuda.mem_get_info()[0] == free
+        check(1.0)
+        if not graph:
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g):
+                assert plan.execute(torch.cuda.current_stream()) == 1
+            for scale in (2.0, 0.5, 4.0):
+                fill(buf, scale)
+                y.fill_(-7.0)
+                g.replay()
+                torch.cuda.synchronize()
+                check(scale)
+        plan.close()
+
