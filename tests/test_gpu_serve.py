@@ -197,3 +197,33 @@ def test_ticket_ring_wraps(torch, C, ctx):
         assert srv.query(0) == 1 and srv.query(count - 1) == 1 and srv.wait(1) == 1
         assert srv.query(count) == -1                   # not issued yet
     assert np.array_equal(y.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("log_max,sizes", [(17, [("cfwd", 1 << 16), ("cinv", 1 << 16), ("cfwd", 1 << 17), ("rfwd", 1 << 17),
+                                                  ("rinv", 1 << 17)]),
+                                           (24, [("cfwd", 1 << 24), ("rinv", 1 << 18)])])   # above the slots' 64 MiB, and below
+def test_requests_with_overlapping_buffers(torch, C, log_max, sizes):
+    """Multi-pass requests whose input and output overlap (intermediates in the slots' buffers, or allocated above
+    64 MiB) beside the same transforms with separate buffers."""
+    with C.Context(1 << log_max) as c:
+        ins, outs, descs = build(torch, C, c, sizes, 11000)
+        wants = [plain(torch, c, kind, n, x) for (kind, n), x in zip(sizes, ins)]
+        bufs, gots = [], []
+        for (kind, n), x, want, d in zip(sizes, ins, wants, list(descs)):
+            half = x.numel() // 4 * 2
+            buf = torch.zeros(max(x.numel(), half + want.numel()), device="cuda")
+            bufs.append(buf)
+            gots.append(buf[half:half + want.numel()])
+            descs.append((d[0], n, buf, gots[-1]))
+        with C.Server(c, 4 << 30, max_in_flight=2) as srv:
+            for _ in range(3):
+                for buf, x in zip(bufs, ins):
+                    buf[:x.numel()] = x.flatten()
+                for y in outs:
+                    y.zero_()
+                torch.cuda.synchronize()
+                srv.replay(descs, np.zeros(len(descs)))
+                assert srv.drain() == 1
+                for i, want in enumerate(wants):
+                    assert torch.equal(outs[i].flatten().view(torch.int32), want.flatten().view(torch.int32)), (i, "separate")
+                    assert torch.equal(gots[i].view(torch.int32), want.flatten().view(torch.int32)), (i, "overlapping")

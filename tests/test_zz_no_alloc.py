@@ -148,3 +148,24 @@ def test_noalloc_rejects_what_does_not_fit(torch, C, ctx):
         assert fwd_only.transform_batch_noalloc(KIND["cinv"], 1024, 1, a, b) == 0
         assert fwd_only.transform_batch_noalloc(KIND["cfwd"], 1024, 1, a, b) == 1
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("kind,first,second", CASES[:4], ids=[c[0] for c in CASES[:4]])
+def test_noalloc_overlapping_buffers(torch, C, ctx, kind, first, second):
+    """Input and output that overlap: the intermediate lies in the fixed scratch, two calls in a row on it, the
+    second smaller.  The bits of separate buffers, and no device memory taken."""
+    for seed, (n, count) in enumerate((first, second)):
+        xt = make_input(torch, kind, n, count, 400 + seed)
+        want = batched(torch, ctx, kind, n, count, xt)
+        half = xt.numel() // 4 * 2                       # whole complex values
+        buf = torch.full((max(xt.numel(), half + want.numel()),), float("nan"), device="cuda")
+        buf[:xt.numel()] = xt.flatten()
+        got = buf[half:half + want.numel()]
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        assert ctx.transform_batch_noalloc(KIND[kind], n, count, buf, got) == 1
+        torch.cuda.synchronize()
+        assert torch.cuda.mem_get_info()[0] == free
+        assert torch.equal(got.view(torch.int32), want.flatten().view(torch.int32)), (n, count)
+        before = buf[:half].clone()                       # what lies before the output stays
+        assert torch.equal(before, xt.flatten()[:half])
