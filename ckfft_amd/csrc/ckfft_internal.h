@@ -37,8 +37,7 @@ constexpr int kLogMaxSupported = kLogMaxPyramid + kLogFine;
 constexpr int kLogXtwCols = 8;
 constexpr int kLogMinXtw = 12;        // tables the library allocates
 constexpr int kLogMinXtwArena = 15;   // tables in a caller's arena, whose size the caller may keep
-// Radix range of one multi-pass stage.
-constexpr int kLogMinPass = 6;
+// Largest radix of one multi-pass stage.
 constexpr int kLogMaxPass = 11;
 
 // Device twiddle tables of a context.
