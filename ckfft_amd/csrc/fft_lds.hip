@@ -146,9 +146,11 @@ constexpr int staged_min(int kind, int logn)
 // 5.5 -> 4.4, complex 1024 x 16384 46.9 -> 45.0).  In the staged kernel no wave waits for another's copies
 // (real forward 512 x 40001 38 -> 35 us, x 65536 54 -> 49, 256 x 10000 7.6 -> 6.7; complex 64 x 199999, forward and
 // inverse, 73.1 -> 70.3); longer real forwards keep 256 there, where 64 gained 5 % at 2^24 points and lost 5 % at 2^21.
-// Where the forward of a real size has 256, its inverse has too for such batches: transforms are dealt
-// to workgroups, and so to XCDs, alike, and an inverse right after a forward finds the spectrum in its own
-// L2 (forward and inverse of 1024 x 4096 16 us, with unequal workgroups 19).
+// Real inverses of 2^8 to 2^10 points have 256 too for such batches.  Where the forward has, transforms are dealt
+// to workgroups, and so to XCDs, alike, and an inverse right after it finds the spectrum in its own
+// L2 (forward and inverse of 1024 x 4096 16 us, with unequal workgroups 19); by itself the inverse of 512 is faster so
+// as well from about 10000 (one wave / 256 threads: x 8192 8.2 / 8.4 us, x 12000 10.8 / 10.2, x 40001 35.6 / 35.0,
+// x 65536 54.7 / 53.5, x 131072 105.4 / 100.9).
 constexpr int plain_wg(int logn, int t) { return t >= 256 ? t : logn >= 5 && logn <= 10 ? (t > 64 ? t : 64) : 256; }
 constexpr int staged_wg(int kind, int logn) { return logn >= 5 && logn <= (kind == kRealForward ? 8 : 7) ? 64 : 256; }
 
@@ -192,8 +194,7 @@ constexpr LaunchCfg make_cfg()
             c.many_wg = SWG;
             c.many_tpw = SWG / T;
             c.many_min = staged_min(KIND, LOGN);
-        } else if constexpr (KIND == kRealInverse && staged_out(kRealForward, LOGN) &&
-                             staged_wg(kRealForward, LOGN) != WG && T < 256) {
+        } else if constexpr (KIND == kRealInverse && staged_out(kRealForward, LOGN) && WG < 256) {
             c.many = fft_lds_kernel<LOGN, LOGP, 256, KIND, SPLIT>;   // not staged, see plain_wg
             c.many_wg = 256;
             c.many_tpw = 256 / T;

@@ -92,7 +92,7 @@ def test_few_signals_of_one_workgroup_size(torch, ctx, kind):  # noqa: F811
         torch.cuda.synchronize()
         assert torch.equal(y.view(count, length).view(torch.int32), want[:count].view(torch.int32)), count
         assert bool((buf[:1024] == -7.0).all()) and bool((buf[-1024:] == -7.0).all()) and torch.equal(xt, kept)
-    # host buffers: the intermediate is the staging slot's device buffer
+    # host buffers: one workgroup
     fn = {"cfwd": ctx.complex_forward, "cinv": ctx.complex_inverse, "rfwd": ctx.real_forward}.get(kind)
     yh = np.zeros(length, np.float32)
     assert (fn(n, x[3], yh) if fn else ctx.real_inverse(n, x[3], yh, np.zeros(n + 2, np.float32))) == 1

@@ -18,7 +18,7 @@ def test_short_batches(torch, ctx, kind, log2n):  # noqa: F811
     n = 1 << log2n
     if kind in ("rfwd", "rinv") and log2n < 3:
         pytest.skip("closed form")
-    # 4096 complex points to a workgroup: 513 workgroups, the last with one signal
+    # 512 times 4096 complex points, whole workgroups of any size, and one signal more
     logc = log2n - 1 if kind in ("rfwd", "rinv") else log2n
     per = 256 * min(16, 1 << logc) >> logc
     count = 512 * per + 1
