@@ -72,8 +72,10 @@ OutputRange output_range(const CkFftBatchDesc& d);
 bool batch_build(const CkFftContext* ctx, const CkFftBatchDesc* descs, int count, int var_override,
                  bool check_pointers, BatchBuild& out, bool narrow);
 // The table pass launches (fft_pass.hip): pass 1 then pass 2 over the n_fwd forward transforms
-// of d_trs followed by its n_inv inverse ones, the intermediate of each in its output.
-hipError_t launch_pass_table(const BatchTransform* d_trs, int n_fwd, int n_inv, const DeviceTables& tb, hipStream_t s);
+// of d_trs followed by its n_inv inverse ones, the intermediate of each in its output; in equal groups
+// of up to `group` transforms, one pair of launches each.
+hipError_t launch_pass_table(const BatchTransform* d_trs, int n_fwd, int n_inv, int group, const DeviceTables& tb,
+                             hipStream_t s);
 // The same with the transforms passed by value, any number of them.
 hipError_t launch_pass_inline(const std::vector<BatchTransform>& fwd, const std::vector<BatchTransform>& inv,
                               const DeviceTables& tb, hipStream_t s);

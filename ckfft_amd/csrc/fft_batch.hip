@@ -527,6 +527,12 @@ bad:
 }
 
 constexpr int kPassesFirst = 512;   // complex 2^16 transforms of a plan from which their passes go first
+// Transforms of one pair of pass launches where they go first: 160 MiB of intermediates, which the second launch finds
+// in the 256 MiB Infinity Cache.  Over all of a plan's 953 transforms at once the pair took 354 us (341 with
+// intermediates in a buffer of their own), in equal groups of up to 128 357, 192 338, 256 336, 320 326, 384 326, 512 331;
+// the plan of 20,000 transforms that holds them 776 us, and 796, 787, 768, 758, 760, 767.  Behind the persistent
+// kernels the passes are one pair: a plan of 10000 (450 passes) takes 369 us, in two groups 381.
+constexpr int kPassGroup = 320;
 
 // The plan's launches that a graph can hold, as three branches that run side by side: the
 // table passes, the narrow persistent launch and the wide one.  With the wide launch alone in
@@ -551,10 +557,13 @@ hipError_t launch_plan_kernels(CkFftBatchPlan* p, hipStream_t s)
     // instead: their tiles then have the chip to themselves, where beside persistent
     // workgroups both are slower.  Mixes of 2^6 .. 2^16 points, passes first / persistent kernels first: 150
     // transforms 72 / 62 us, 400 79 / 65, 1070 88 / 78, 4000 178 / 174, 10000 (about 450 of them 2^16) 372 / 368,
-    // 13000 (590) 468 / 488, 20000 708 / 751.
+    // 13000 (590) 466 / 488, 20000 699 / 751 (executions over one set of buffers; over changing ones 720).
     const bool passes_first = p->n_pass_fwd + p->n_pass_inv >= kPassesFirst;
     hipError_t e = hipSuccess;
-    if (passes_first) e = launch_pass_table(p->d_pass, p->n_pass_fwd, p->n_pass_inv, tb, s_pass);
+    const auto passes = [&]() {
+        return launch_pass_table(p->d_pass, p->n_pass_fwd, p->n_pass_inv, passes_first ? kPassGroup : kPassesFirst, tb, s_pass);
+    };
+    if (passes_first) e = passes();
     const auto wide = [&]() {
         return p->n_wide ? launch_persistent_raw(p->d_items, p->n_wide, p->d_trs, p->d_ctl, p->grid, tb, s, false)
                          : hipSuccess;
@@ -563,7 +572,7 @@ hipError_t launch_plan_kernels(CkFftBatchPlan* p, hipStream_t s)
     if (e == hipSuccess && p->n_items > p->n_wide)
         e = launch_persistent_raw(p->d_items + p->n_wide, p->n_items - p->n_wide, p->d_trs, p->d_ctl + kCtlWords,
                                   p->grid_narrow, tb, s_narrow, true);
-    if (e == hipSuccess) e = passes_first ? wide() : launch_pass_table(p->d_pass, p->n_pass_fwd, p->n_pass_inv, tb, s_pass);
+    if (e == hipSuccess) e = passes_first ? wide() : passes();
     if (branches)
         for (int i = 0; i < 2; ++i) {
             fe = hipEventRecord(p->join[i], p->branch[i]);

@@ -212,3 +212,28 @@ def test_plan_of_overlapping_buffers(torch, C, graph):  # noqa: F811
                 check(scale)
         plan.close()
 
+
+
+@pytest.mark.parametrize("passes", [512, 640, 641])
+def test_plan_pass_groups(torch, C, passes):  # noqa: F811
+    """Plans whose 2^16 transforms take two and three pairs of table launches, with directions that change
+    within a group: the bits of the stand-alone calls."""
+    n, distinct = 1 << 16, 7
+    gen = torch.Generator(device="cuda").manual_seed(0x320 + passes)
+    x = torch.randn((distinct, 2 * n), device="cuda", generator=gen)
+    want = torch.empty((2, distinct, 2 * n), device="cuda")
+    with C.Context(n) as c:
+        assert c.complex_forward_batch(n, distinct, x, want[0]) == 1
+        assert c.complex_inverse_batch(n, distinct, x, want[1]) == 1
+        y = torch.full((passes, 2 * n), -7.0, device="cuda")
+        kinds = [i % 3 == 0 for i in range(passes)]            # a third inverse
+        plan = C.BatchPlan(c, [(C.kCkFftKind_ComplexInverse if kinds[i] else C.kCkFftKind_ComplexForward, n, x[i % distinct],
+                                y[i]) for i in range(passes)], graph=True)
+        assert plan.info()["pass_transforms"] == passes
+        for _ in range(2):
+            y.fill_(-7.0)
+            assert plan.execute(torch.cuda.current_stream()) == 1
+            torch.cuda.synchronize()
+            for i in range(passes):
+                assert torch.equal(y[i].view(torch.int32), want[int(kinds[i])][i % distinct].view(torch.int32)), i
+        plan.close()
