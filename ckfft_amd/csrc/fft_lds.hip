@@ -130,13 +130,17 @@ constexpr bool staged_out(int kind, int logn) { return logn >= 2 && logn <= (kin
 
 // Transforms from which the staged kernel is taken (below, the plain one: the two extra passes
 // through LDS cost 0.3-1 us of latency, which only a batch that fills the chip gets back).
-// One-thread transforms always: their plain reads touch one 8-byte value per line.  Measured
+// One-thread transforms always, their plain reads touch one 8-byte value per line, but for the real inverse of 8
+// samples, whose lines the threads of a wave share.  Measured
 // crossings, plain against staged: complex 2^7 8.2 / 8.2 us x 8192 and 14.6 / 11.7 x 16384;
-// real forward 2^7 points 5.9 / 5.7 x 2048, 2^9 7.4 / 7.2 x 2048 and 10.7 / 9.3 x 4096; real inverse
-// 2^8 samples 6.9 / 7.1 x 8192 and 10.3 / 9.4 x 16384.
+// real forward 2^7 points 5.9 / 5.7 x 2048, 2^9 7.4 / 7.2 x 2048 and 10.7 / 9.3 x 4096, 2^11 9.9 / 11.0 x 1300, 12.7 / 12.7
+// x 1800 and 14.9 / 12.8 x 2048; real inverse 2^8 samples 6.9 / 7.1 x 8192 and 10.3 / 9.4 x 16384, 8 samples 5.0 / 5.7
+// x 300000, 5.9 / 7.0 x 400000, 7.7 / 7.5 x 450000 and 8.7 / 8.1 x 524288.
 constexpr int staged_min(int kind, int logn)
 {
+    if (kind == kRealInverse && logn == 2) return 13 << 15;
     if (logn <= 4) return 0;
+    if (kind == kRealForward && logn == 11) return 7 << 8;
     const int log_points = kind == kRealForward ? (logn <= 7 ? 18 : 21) : logn <= 5 ? 18 : logn == 6 ? 19 : 21;
     return 1 << (log_points - logn);
 }
@@ -146,12 +150,13 @@ constexpr int staged_min(int kind, int logn)
 // 5.5 -> 4.4, complex 1024 x 16384 46.9 -> 45.0).  In the staged kernel no wave waits for another's copies
 // (real forward 512 x 40001 38 -> 35 us, x 65536 54 -> 49, 256 x 10000 7.6 -> 6.7; complex 64 x 199999, forward and
 // inverse, 73.1 -> 70.3); longer real forwards keep 256 there, where 64 gained 5 % at 2^24 points and lost 5 % at 2^21.
-// Real inverses of 2^8 to 2^10 points have 256 too for such batches.  Where the forward has, transforms are dealt
-// to workgroups, and so to XCDs, alike, and an inverse right after it finds the spectrum in its own
-// L2 (forward and inverse of 1024 x 4096 16 us, with unequal workgroups 19); by itself the inverse of 512 is faster so
-// as well from about 10000 (one wave / 256 threads: x 8192 8.2 / 8.4 us, x 12000 10.8 / 10.2, x 40001 35.6 / 35.0,
-// x 65536 54.7 / 53.5, x 131072 105.4 / 100.9).
+// Real inverses of 2^9 and 2^10 points have 256 too for such batches: transforms are dealt
+// to workgroups, and so to XCDs, alike, and an inverse right after its forward finds the spectrum in its own
+// L2 (forward and inverse of 1024 x 4096 16 us, with unequal workgroups 19).  Those of 2^8 have 256 from 11264 on
+// (one wave / 256 threads: x 10000 8.9 / 10.6 us, x 12000 10.9 / 10.2, x 40001 35.6 / 35.0, x 65536 54.7 / 53.5,
+// x 131072 105.4 / 100.9).
 constexpr int plain_wg(int logn, int t) { return t >= 256 ? t : logn >= 5 && logn <= 10 ? (t > 64 ? t : 64) : 256; }
+constexpr int wide_inverse_min(int logn) { return logn == 8 ? 11 << 10 : staged_min(kRealForward, logn); }
 constexpr int staged_wg(int kind, int logn) { return logn >= 5 && logn <= (kind == kRealForward ? 8 : 7) ? 64 : 256; }
 
 template <int LOGN, int KIND>
@@ -198,7 +203,7 @@ constexpr LaunchCfg make_cfg()
             c.many = fft_lds_kernel<LOGN, LOGP, 256, KIND, SPLIT>;   // not staged, see plain_wg
             c.many_wg = 256;
             c.many_tpw = 256 / T;
-            c.many_min = staged_min(kRealForward, LOGN);
+            c.many_min = wide_inverse_min(LOGN);
         }
         return c;
     }

@@ -292,9 +292,10 @@ hipError_t staged_transform(StagingPool* pool, Kind kind, int log2n, const void*
         // the calling thread's own default stream: calls from several threads sharing a
         // context (inc/ckfft/ckfft.h:39-41) overlap on the device instead of queueing on
         // the null stream, which they still follow as a blocking stream does
-        // A complex transform of 2^15 points stays one workgroup and one launch here: eight threads then
-        // finish 320 calls in 0.37 of one thread's time (3.6 of 9.5 ms), while with the two launches
-        // one thread takes 6.5 ms and eight 3.3 ms, bound by the host's launches and waits.
+        // A complex transform of 2^15 points stays one workgroup and one launch here.  With two launches one
+        // caller is faster (320 calls 6.5 ms against 9.5) and eight threads about equal (3.2 ms against 3.4), bound by
+        // the host's launches and waits, so calls of different threads overlap less: eight threads take 0.36
+        // of one thread's time now and would take 0.5, 0.75 at times; tests/test_gpu_parity.py holds them to 0.7.
         const bool spread = kind == kRealForward || kind == kRealInverse;
         hipError_t e = launch_transform(kind, log2n, 1, in, out, tb, hipStreamPerThread, nullptr, 0, spread);
         return e != hipSuccess ? e : hipStreamSynchronize(hipStreamPerThread);

@@ -192,3 +192,32 @@ def test_workgroup_sizes(torch, ctx, kind, log2c):  # noqa: F811
             assert O.split_norm_err(got, oracle_out(kind, n, x)) <= TOL_REF
             assert O.rel_l2(got, fp64_out(kind, n, x)) <= TOL_FP64
         assert torch.equal(y.view(torch.int32), first[rows].view(torch.int32))
+
+
+# (kind, size, split mode, count): batch sizes from which another kernel is taken
+@pytest.mark.parametrize("kind,log2n,split,least", [("rfwd", 12, False, 7 << 8), ("rinv", 9, False, 11 << 10),
+                                                     ("rinv", 3, False, 13 << 15)])
+def test_either_side_of_a_rule(torch, C, kind, log2n, split, least):  # noqa: F811
+    n, distinct = 1 << log2n, 9
+    x = make_input(kind, n, distinct, 0x71 + log2n)
+    xt = torch.from_numpy(x).cuda()
+    length, guard, first = out_len(kind, n), 64, None
+    with C.Context(n, C.kCkFftDirection_Both) as c:
+        assert not split or c.set_precision(C.kCkFftPrecision_SplitBf16x3) == 1
+        fn = {"cfwd": c.complex_forward_batch, "cinv": c.complex_inverse_batch, "rfwd": c.real_forward_batch,
+              "rinv": c.real_inverse_batch}[kind]
+        for count in (distinct, least - 1, least, least + 1):
+            rows = torch.arange(count, device="cuda") % distinct
+            xin = xt[rows].contiguous()
+            buf = torch.full((guard + count * length + guard,), -7.0, device="cuda")
+            y = buf[guard:guard + count * length]
+            assert fn(n, count, xin, y) == 1
+            torch.cuda.synchronize()
+            assert bool((buf[:guard] == -7.0).all()) and bool((buf[-guard:] == -7.0).all())
+            y = y.view(count, length)
+            if first is None:
+                first = y.clone()
+                got = first.cpu().numpy()
+                assert O.split_norm_err(got, oracle_out(kind, n, x)) <= TOL_REF
+                assert O.rel_l2(got, fp64_out(kind, n, x)) <= TOL_FP64
+            assert torch.equal(y.view(torch.int32), first[rows].view(torch.int32))
