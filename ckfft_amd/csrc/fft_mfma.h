@@ -270,9 +270,10 @@ struct SignalIO {
 // the exchange changed nothing): span 16 a copy in LDS
 // (w16[16 q + m]), span 256 the context's transposed table (level 2^log_xtw >= 2^12, row q of level
 // 2^12 at q << (log_xtw - 12)).  The values are the pyramid's bits.  XTW: the context has that table.
-template <bool XTW>
+// W16: the kernel has the copy of span 16.
+template <bool XTW, bool W16>
 struct MfmaTwiddles {
-    static constexpr bool kXtw = XTW;
+    static constexpr bool kXtw = XTW, kW16 = W16;
     const float2* __restrict__ pyr;
     const float2* w16;                   // LDS, 256 values (fill_w16), or unused
     const float2* __restrict__ xtw;
@@ -345,7 +346,7 @@ __device__ __forceinline__ void mfma_stage(const SRC& src, const DST& dst, const
         src.template load<8, NB>(f / NB, i + 8 * h * NB, x);
         if constexpr (NS > 1) {
             const int m = i & (NS - 1);
-            if constexpr (NS == 16) {
+            if constexpr (NS == 16 && TW::kW16) {
                 const float2* tw = tws.w16 + 128 * h + m;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) x[e] = cmul(x[e], dirw<INV>(tw[16 * e]));

@@ -28,12 +28,14 @@ struct WholeShape {
     using TL = MfmaTile<LOGN, LOGB>;
 };
 
+constexpr bool has_span16(int logn) { return logn % 4 == 0 ? logn >= 8 : logn == 13; }
+
 // The first stage reads the signals straight from global memory and the last writes
 // them back; the stages between exchange through the LDS tile.  Short signals are copied to
 // and from the tile in memory order instead, whole lines a wave (2^24 points: n = 16 125 -> 49 us,
 // 32 137 -> 53, 64 100 -> 52; 128 and above were no faster so), if the batch has staged_min_groups
-// workgroups.
-template <int LOGN, bool INV, bool STAGED, bool XTW>
+// workgroups.  W16: the stage of span 16 reads its twiddles from a copy in LDS.
+template <int LOGN, bool INV, bool STAGED, bool XTW, bool W16>
 __global__ __launch_bounds__(WholeShape<LOGN>::WG) void fft_mfma_whole_kernel(const float2* __restrict__ in,
                                                                               float2* __restrict__ out,
                                                                               const float2* __restrict__ pyr,
@@ -43,13 +45,12 @@ __global__ __launch_bounds__(WholeShape<LOGN>::WG) void fft_mfma_whole_kernel(co
     using SH = WholeShape<LOGN>;
     using TL = typename SH::TL;
     constexpr int STAGES = (LOGN % 4 ? 1 : 0) + LOGN / 4, WG = SH::WG;
-    // the stage of span 16, if any (the first stage's barrier comes before its use)
-    constexpr bool W16 = LOGN % 4 == 0 ? LOGN >= 8 : LOGN == 13;
+    static_assert(!W16 || has_span16(LOGN), "no stage of span 16");
     __shared__ float2 lds[STAGES > 1 || STAGED ? TL::WORDS : 1];
     __shared__ float2 w16[W16 ? 256 : 1];
     const int tid = threadIdx.x;
-    if constexpr (W16) fill_w16(w16, pyr, tid);
-    const MfmaTwiddles<XTW> tws{pyr, w16, xtw, log_xtw};
+    if constexpr (W16) fill_w16(w16, pyr, tid);   // the first stage's barrier comes before its use
+    const MfmaTwiddles<XTW, W16> tws{pyr, w16, xtw, log_xtw};
     const long long g0 = (long long)blockIdx.x << SH::LOGB;
     if constexpr (STAGED) {
         constexpr int POINTS = TL::B << LOGN, K = POINTS / WG;
@@ -124,7 +125,7 @@ __global__ __launch_bounds__(512) void fft_mfma_pass_kernel(const float2* in, fl
     }
     __syncthreads();
     const LdsIO<TL> lio{lds};
-    mfma_columns_fft<TL, WG, INV>(lio, lio, lio, MfmaTwiddles<false>{pyr, w16, nullptr, 0}, tid);
+    mfma_columns_fft<TL, WG, INV>(lio, lio, lio, MfmaTwiddles<false, LOGR == 8>{pyr, w16, nullptr, 0}, tid);
     if constexpr (FIRST) {
 #pragma unroll 4
         for (int e = tid; e < T; e += WG) {
@@ -151,13 +152,19 @@ using WholeFn = void (*)(const float2*, float2*, const float2*, const float2*, i
 // x 4096 (16) and 4.8 / 4.3 x 30000 (118).
 constexpr long long staged_min_groups(int logn) { return logn == 4 ? 0 : logn == 5 ? 144 : logn == 6 ? 208 : 1ll << 31; }
 
+// Workgroups from which 2^8 points (one exchange, 16 signals to a workgroup) read the twiddles of span 16 from the copy in
+// LDS; below, its fill costs more than the pyramid's gather.  us forward and inverse, pyramid / copy: x 11718 24.0 / 24.8,
+// x 23437 42.3 / 45.5, x 27144 48.0 / 52.7, x 32768 54.8 / 55.6, x 65536 99.0 / 95.1.
+constexpr long long kW16MinGroups = 3072;
+
 // XTW only where a stage of span 256 is a matrix-core one: 2^12 and 2^13 points.
-template <int LOGN, bool STAGED>
+template <int LOGN, bool STAGED, bool W16>
 static WholeFn whole_fn(bool inv, bool xtw)
 {
     constexpr bool X = LOGN == 12 || LOGN == 13;
-    if (xtw) return inv ? fft_mfma_whole_kernel<LOGN, true, STAGED, X> : fft_mfma_whole_kernel<LOGN, false, STAGED, X>;
-    return inv ? fft_mfma_whole_kernel<LOGN, true, STAGED, false> : fft_mfma_whole_kernel<LOGN, false, STAGED, false>;
+    if (xtw)
+        return inv ? fft_mfma_whole_kernel<LOGN, true, STAGED, X, W16> : fft_mfma_whole_kernel<LOGN, false, STAGED, X, W16>;
+    return inv ? fft_mfma_whole_kernel<LOGN, true, STAGED, false, W16> : fft_mfma_whole_kernel<LOGN, false, STAGED, false, W16>;
 }
 
 template <int LOGN>
@@ -165,11 +172,13 @@ static WholeFn whole_fn(bool inv, bool xtw, long long groups)
 {
     constexpr long long from = staged_min_groups(LOGN);
     if constexpr (from == 0)
-        return whole_fn<LOGN, true>(inv, xtw);
+        return whole_fn<LOGN, true, false>(inv, xtw);
+    else if constexpr (LOGN == 8)
+        return groups >= kW16MinGroups ? whole_fn<LOGN, false, true>(inv, xtw) : whole_fn<LOGN, false, false>(inv, xtw);
     else if constexpr (from > 0x7fffffffll)
-        return whole_fn<LOGN, false>(inv, xtw);
+        return whole_fn<LOGN, false, has_span16(LOGN)>(inv, xtw);
     else
-        return groups >= from ? whole_fn<LOGN, true>(inv, xtw) : whole_fn<LOGN, false>(inv, xtw);
+        return groups >= from ? whole_fn<LOGN, true, false>(inv, xtw) : whole_fn<LOGN, false, false>(inv, xtw);
 }
 
 static WholeFn whole_kernel(int logn, bool inv, bool xtw, long long count, int* wg, long long* groups)

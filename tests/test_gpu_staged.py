@@ -196,7 +196,8 @@ def test_workgroup_sizes(torch, ctx, kind, log2c):  # noqa: F811
 
 # (kind, size, split mode, count): batch sizes from which another kernel is taken
 @pytest.mark.parametrize("kind,log2n,split,least", [("rfwd", 12, False, 7 << 8), ("rinv", 9, False, 11 << 10),
-                                                     ("rinv", 3, False, 13 << 15)])
+                                                     ("rinv", 3, False, 13 << 15), ("cfwd", 8, True, 3071 * 16 + 1),
+                                                     ("cinv", 8, True, 3071 * 16 + 1)])
 def test_either_side_of_a_rule(torch, C, kind, log2n, split, least):  # noqa: F811
     n, distinct = 1 << log2n, 9
     x = make_input(kind, n, distinct, 0x71 + log2n)
