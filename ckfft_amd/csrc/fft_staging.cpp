@@ -43,7 +43,7 @@ constexpr size_t kKeepBytes = (size_t)256 << 20;
 // forward (real: 8n + 256 bytes and 8n + 8), finds room in the forward's: freeing and allocating them
 // again took most of a context's second call (real 1024 54 us, now 14; 65536 106 / 56; 2^18 232 / 160).
 constexpr size_t kGrowBytes = (size_t)64 << 10;
-constexpr size_t kMinChunk = 1 << 20;   // bytes per pipelined copy chunk (at least)
+constexpr size_t kMinChunk = 1 << 20;   // bytes per pipelined copy chunk (at least, if there are several)
 constexpr int kMaxChunks = 16;
 
 struct Slot {
@@ -58,20 +58,25 @@ struct Slot {
 
 enum MemKind { kHostPageable, kHostPinned, kDevice };
 
-// own: device memory of the current device itself, neither managed nor another device's.
-MemKind classify(const void* p, bool* own = nullptr)
+// device: the device of plain device memory, -1 for any other (managed memory is kDevice too).
+MemKind classify(const void* p, int* device = nullptr)
 {
     hipPointerAttribute_t a;
-    if (own) *own = false;
+    if (device) *device = -1;
     if (hipPointerGetAttributes(&a, p) != hipSuccess) {
         (void)hipGetLastError();   // plain pageable host memory is unknown to HIP
         return kHostPageable;
     }
-    int device = -1;
-    if (own && a.type == hipMemoryTypeDevice) *own = hipGetDevice(&device) == hipSuccess && a.device == device;
+    if (device && a.type == hipMemoryTypeDevice) *device = a.device;
     if (a.type == hipMemoryTypeDevice || a.type == hipMemoryTypeManaged) return kDevice;
     if (a.type == hipMemoryTypeHost) return kHostPinned;
     return kHostPageable;
+}
+
+bool on_current(int device)
+{
+    int current = -1;
+    return device >= 0 && hipGetDevice(&current) == hipSuccess && current == device;
 }
 
 void free_slot(Slot* s)
@@ -85,11 +90,12 @@ void free_slot(Slot* s)
     delete s;
 }
 
-// Chunk layout of `bytes`: at most kMaxChunks chunks of at least kMinChunk, 256-aligned.
+// Chunk layout of `bytes`: equal chunks, as many as there are whole kMinChunk up to kMaxChunks, 256-aligned (a real
+// forward's 8 bytes above a power of two had a chunk of their own: real 2^19 from pinned memory 202 us, now 168).
 size_t chunk_size(size_t bytes)
 {
-    size_t c = std::max(kMinChunk, (bytes + kMaxChunks - 1) / kMaxChunks);
-    return (c + 255) & ~size_t(255);
+    const size_t chunks = std::min((size_t)kMaxChunks, std::max((size_t)1, bytes / kMinChunk));
+    return ((bytes + chunks - 1) / chunks + 255) & ~size_t(255);
 }
 
 }  // namespace
@@ -199,7 +205,7 @@ bool reported(const Slot* s)
     }
 }
 
-hipError_t run_direct(Slot* s, Kind kind, int log2n, const void* in, size_t ib, MemKind kin, bool own, void* out,
+hipError_t run_direct(Slot* s, Kind kind, int log2n, const void* in, size_t ib, MemKind kin, int in_device, void* out,
                       size_t ob, MemKind kout, const DeviceTables& tb)
 {
     const size_t ib_al = (ib + 255) & ~size_t(255);
@@ -211,7 +217,7 @@ hipError_t run_direct(Slot* s, Kind kind, int log2n, const void* in, size_t ib, 
     // memory, and the current device's own memory every launch reads as it is; a caller's pinned memory may
     // be non-coherent, so it is copied (real 1024, pinned to pageable: 10.6 us a call in place, 10.8 copied, 17.3
     // with the wait), and managed memory or another device's waits for the stream.
-    const bool word = kout == kHostPageable && signal_supported(kind, log2n) && (kin != kDevice || own);
+    const bool word = kout == kHostPageable && signal_supported(kind, log2n) && (kin != kDevice || on_current(in_device));
     if (kin == kHostPageable || (word && kin == kHostPinned)) {
         std::memcpy(s->h_buf, in, ib);
         src = s->h_buf;
@@ -235,22 +241,24 @@ hipError_t run_direct(Slot* s, Kind kind, int log2n, const void* in, size_t ib, 
     return e;
 }
 
-hipError_t run_staged(Slot* s, Kind kind, int log2n, const void* in, size_t ib, MemKind kin, bool own, void* out,
+hipError_t run_staged(Slot* s, Kind kind, int log2n, const void* in, size_t ib, MemKind kin, int in_device, void* out,
                       size_t ob, MemKind kout, const DeviceTables& tb)
 {
     const size_t ib_al = (ib + 255) & ~size_t(255);
     hipError_t e = grow(s, ib_al + ob);
     if (e != hipSuccess) return e;
-    if (one_pass(kind, log2n, tb)) return run_direct(s, kind, log2n, in, ib, kin, own, out, ob, kout, tb);
+    if (one_pass(kind, log2n, tb)) return run_direct(s, kind, log2n, in, ib, kin, in_device, out, ob, kout, tb);
     char* d_in = s->d_buf;
     char* d_out = s->d_buf + ib_al;
     // input
     const void* src = in;
+    bool flush = false;   // the input came in several chunks
     if (kin == kHostPinned) {
         e = hipMemcpyAsync(d_in, in, ib, hipMemcpyHostToDevice, s->stream);
         src = d_in;
     } else if (kin == kHostPageable) {
         const size_t cs = chunk_size(ib);
+        flush = ib > cs;
         for (size_t off = 0; off < ib && e == hipSuccess; off += cs) {
             const size_t len = std::min(cs, ib - off);
             std::memcpy(s->h_buf + off, (const char*)in + off, len);
@@ -260,6 +268,10 @@ hipError_t run_staged(Slot* s, Kind kind, int log2n, const void* in, size_t ib, 
     }
     void* dst = kout == kDevice ? out : (void*)d_out;
     if (e == hipSuccess) e = launch_transform(kind, log2n, 1, src, dst, tb, s->stream);
+    // Several copies up, the kernels and several copies down, queued with no look at the stream in between, wait for each
+    // other longer: complex 2^18 (2 MiB each way, two chunks) 236 us forward, with this query 205; real 2^19
+    // 232 / 207.  Larger calls are the same either way; calls of one chunk lose 4-6 us by it.
+    if (e == hipSuccess && flush && kout == kHostPageable) (void)hipStreamQuery(s->stream);
     // output
     if (e == hipSuccess && kout == kHostPinned) {
         e = hipMemcpyAsync(out, d_out, ob, hipMemcpyDeviceToHost, s->stream);
@@ -286,8 +298,8 @@ hipError_t run_staged(Slot* s, Kind kind, int log2n, const void* in, size_t ib, 
 hipError_t staged_transform(StagingPool* pool, Kind kind, int log2n, const void* in, size_t ib, void* out, size_t ob,
                             const DeviceTables& tb)
 {
-    bool own = false;
-    const MemKind kin = classify(in, &own), kout = classify(out);
+    int in_device = -1;
+    const MemKind kin = classify(in, &in_device), kout = classify(out);
     if (kin == kDevice && kout == kDevice) {
         // the calling thread's own default stream: calls from several threads sharing a
         // context (inc/ckfft/ckfft.h:39-41) overlap on the device instead of queueing on
@@ -303,7 +315,7 @@ hipError_t staged_transform(StagingPool* pool, Kind kind, int log2n, const void*
     hipError_t e = hipSuccess;
     Slot* s = acquire(pool, &e);
     if (!s) return e;
-    e = run_staged(s, kind, log2n, in, ib, kin, own, out, ob, kout, tb);
+    e = run_staged(s, kind, log2n, in, ib, kin, in_device, out, ob, kout, tb);
     release(pool, s);
     return e;
 }

@@ -69,6 +69,11 @@ hipError_t hipStreamSynchronize(hipStream_t)
     call("hipStreamSynchronize");
     return hipSuccess;
 }
+hipError_t hipStreamQuery(hipStream_t)
+{
+    call("hipStreamQuery");
+    return hipSuccess;
+}
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned)
 {
     call("hipStreamWaitEvent");

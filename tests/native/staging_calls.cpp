@@ -113,6 +113,18 @@ int main()
     c = one(pool, in.data(), out.data());
     CHECK(c.signal == 1 && c.sync == 0);
     staging_destroy(pool);
+    // pageable calls above one workgroup: the stream is looked at behind the kernels if the input came in several chunks
+    for (int log2n : {17, 18, 19, 20}) {
+        const size_t bytes = (size_t)4 << log2n;
+        std::vector<float> a(1 << log2n, 1.0f), b((1 << log2n) + 2);
+        DeviceTables tb{};
+        StagingPool* p = staging_create();
+        const int before = count_calls("hipStreamQuery");
+        CHECK(staged_transform(p, kRealForward, log2n, a.data(), bytes, b.data(), bytes + 8, tb) == hipSuccess);
+        CHECK(count_calls("hipStreamQuery") - before == (bytes > (1u << 20)));
+        CHECK(b[0] == 2.0f && b[(1 << log2n) - 1] == 2.0f);
+        staging_destroy(p);
+    }
     // a size's inverse finds room in its forward's buffers (real n: 4n in, 4n + 8 out, and the other way round)
     for (int log2n = 4; log2n <= 20; ++log2n) {
         const size_t n = (size_t)1 << log2n;
