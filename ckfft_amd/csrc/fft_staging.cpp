@@ -271,7 +271,8 @@ hipError_t run_staged(Slot* s, Kind kind, int log2n, const void* in, size_t ib, 
     // Several copies up, the kernels and several copies down, queued with no look at the stream in between, wait for each
     // other longer: complex 2^18 (2 MiB each way, two chunks) 236 us forward, with this query 205; real 2^19
     // 232 / 207.  Larger calls are the same either way; calls of one chunk lose 4-6 us by it.
-    if (e == hipSuccess && flush && kout == kHostPageable) (void)hipStreamQuery(s->stream);
+    if (e == hipSuccess && flush && kout == kHostPageable && hipStreamQuery(s->stream) == hipErrorNotReady)
+        (void)hipGetLastError();   // not an error of the next launch
     // output
     if (e == hipSuccess && kout == kHostPinned) {
         e = hipMemcpyAsync(out, d_out, ob, hipMemcpyDeviceToHost, s->stream);

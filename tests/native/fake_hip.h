@@ -52,7 +52,13 @@ static bool await_calls(const std::string& what, int n)
 
 extern "C" {
 hipError_t hipSetDevice(int) { return hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
+static hipError_t fake_last = hipSuccess;
+hipError_t hipGetLastError()
+{
+    const hipError_t e = fake_last;
+    fake_last = hipSuccess;
+    return e;
+}
 const char* hipGetErrorString(hipError_t) { return "error"; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned)
 {
@@ -72,7 +78,7 @@ hipError_t hipStreamSynchronize(hipStream_t)
 hipError_t hipStreamQuery(hipStream_t)
 {
     call("hipStreamQuery");
-    return hipSuccess;
+    return fake_last = hipErrorNotReady;
 }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned)
 {

@@ -122,6 +122,7 @@ int main()
         const int before = count_calls("hipStreamQuery");
         CHECK(staged_transform(p, kRealForward, log2n, a.data(), bytes, b.data(), bytes + 8, tb) == hipSuccess);
         CHECK(count_calls("hipStreamQuery") - before == (bytes > (1u << 20)));
+        CHECK(hipGetLastError() == hipSuccess);
         CHECK(b[0] == 2.0f && b[(1 << log2n) - 1] == 2.0f);
         staging_destroy(p);
     }
